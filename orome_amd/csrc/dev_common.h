@@ -42,6 +42,10 @@ typedef uint32_t u2 __attribute__((ext_vector_type(2)));
     } while (0)
 
 DEV h2 as_h2(uint32_t v) { return __builtin_bit_cast(h2, v); }
+/* fp32 truncated to bf16 (inference/src/format.m:436-450).  The value comes
+ * as a parameter: a bit cast of a vector's element written in place reads the
+ * vector's first element. */
+DEV float bf16_trunc(float v) { return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v) & 0xFFFF0000u); }
 DEV uint32_t as_u32(h2 v) { return __builtin_bit_cast(uint32_t, v); }
 
 DEV float f16_bits_to_f32(uint32_t bits16) {

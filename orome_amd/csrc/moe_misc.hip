@@ -272,10 +272,10 @@ __global__ __launch_bounds__(64 * CN_W) void k_combine_norm(const float *y, cons
             const f4 o = ro[i][lane];
             const f4 wn = nw ? wq[q] : f4{1, 1, 1, 1};
             f4 r;
-            r.x = (o.x * scale) * __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, wn.x) & 0xFFFF0000u);
-            r.y = (o.y * scale) * __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, wn.y) & 0xFFFF0000u);
-            r.z = (o.z * scale) * __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, wn.z) & 0xFFFF0000u);
-            r.w = (o.w * scale) * __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, wn.w) & 0xFFFF0000u);
+            r.x = (o.x * scale) * bf16_trunc(wn.x);
+            r.y = (o.y * scale) * bf16_trunc(wn.y);
+            r.z = (o.z * scale) * bf16_trunc(wn.z);
+            r.w = (o.w * scale) * bf16_trunc(wn.w);
             *(f4 *)(xnorm + (size_t)t * H + j) = r;
             if (x16) /* the GEMMs' fp16 copy, (0,2,1,3) within the 4-group */
                 *(h4 *)(x16 + (size_t)t * H + j) = h4{(_Float16)r.x, (_Float16)r.z, (_Float16)r.y, (_Float16)r.w};

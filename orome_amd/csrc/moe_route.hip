@@ -858,10 +858,10 @@ __global__ __launch_bounds__(64) void k_rmsnorm(const float *h, const float *w, 
             const int j = 256 * i + 4 * lane;
             const f4 wq = w ? wv[i] : f4{1, 1, 1, 1};
             f4 o;
-            o.x = (v[i].x * scale) * __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, wq.x) & 0xFFFF0000u);
-            o.y = (v[i].y * scale) * __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, wq.y) & 0xFFFF0000u);
-            o.z = (v[i].z * scale) * __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, wq.z) & 0xFFFF0000u);
-            o.w = (v[i].w * scale) * __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, wq.w) & 0xFFFF0000u);
+            o.x = (v[i].x * scale) * bf16_trunc(wq.x);
+            o.y = (v[i].y * scale) * bf16_trunc(wq.y);
+            o.z = (v[i].z * scale) * bf16_trunc(wq.z);
+            o.w = (v[i].w * scale) * bf16_trunc(wq.w);
             *(f4 *)(x + (size_t)t * H + j) = o;
         }
 }

@@ -356,10 +356,10 @@ DEV void canon_dots(const float *wrow, const RouteArgs &a, int lane, bool write_
                 if (!wrow) wv[i] = f4{0, 0, 0, 0};
                 if (NORM) {
                     const f4 w = a.norm_w ? nw[i] : f4{1, 1, 1, 1};
-                    nw[i] = f4{__builtin_bit_cast(float, __builtin_bit_cast(uint32_t, w.x) & 0xFFFF0000u),
-                               __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, w.y) & 0xFFFF0000u),
-                               __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, w.z) & 0xFFFF0000u),
-                               __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, w.w) & 0xFFFF0000u)};
+                    nw[i] = f4{bf16_trunc(w.x),
+                               bf16_trunc(w.y),
+                               bf16_trunc(w.z),
+                               bf16_trunc(w.w)};
                 }
             }
         }

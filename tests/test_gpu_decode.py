@@ -379,6 +379,39 @@ def test_stack_prefill_fused_norm():
     p.gm.close()
 
 
+def _norm_weights(img, om):
+    """Norm weights about one, a different one for every element, not bf16 values."""
+    for l in range(om.L):
+        om.norm_weight(l)[:] = 1.0 + 0.25 * orome_amd.synth_normal(92, l, om.H)
+
+
+@pytest.mark.parametrize("T", [1, 2, 5, 40])
+def test_norm_weights(T):
+    """RMSNorm weights that differ from element to element, through each place
+    that normalises: the small-batch router (T <= 16), the norm kernel and the
+    combine that forms the next layer's norm (T = 40).  The second layer's
+    routing is bit-exact against the oracle's norm of the first layer's output."""
+    banner("norm weights, T=%d" % T)
+    p = Pair(layers=2, E=64, seed=92, centered=True, mutate=_norm_weights)
+    h0 = (orome_amd.synth_normal(92, 3, T * p.H) * 4).reshape(T, p.H)
+    dh = DeviceBuffer.from_array(p.ctx, h0)
+    h = h0
+    for l in range(2):
+        p.gm.layer_forward(l, dh, T)
+        p.ctx.sync()
+        got, dbg = dh.download(np.float32, (T, p.H)), p.gm.debug_outputs(T)
+        ref, rdbg = p.om.forward(l, p.om.rmsnorm(l, h), h, debug=True)
+        assert np.array_equal(dbg["idx"], rdbg["idx"])
+        assert_logits(dbg, rdbg)
+        assert rel_l2(got - h, ref - h) < TOL
+        h = got
+    dh2 = DeviceBuffer.from_array(p.ctx, h0)
+    p.gm.stack_forward(dh2, T)
+    p.ctx.sync()
+    assert np.array_equal(dh2.download(np.float32, (T, p.H)), h)
+    p.gm.close()
+
+
 def test_graph_replay_matches_eager(base):
     """Capture three forwards in a HIP graph, replay it several times with eager
     work and synchronisations in between, and check every replay."""
