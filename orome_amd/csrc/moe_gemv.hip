@@ -23,6 +23,8 @@
  * (2590-2668), dequant_matvec_q6k/_q8_0 (1888-1988, 1627-1701) and
  * moe_combine_copy_sq_k8 (1079-1135).
  */
+#include <type_traits>
+
 #include "dev_common.h"
 #include "kernels.h"
 #include "route_dev.h"
@@ -311,23 +313,30 @@ DEV void gu_body(const GUArgs &a, const uint8_t *gbase, const uint8_t *ubase, in
                     glu_f16(red[(i * 2) * 16 + j], red[(i * 2 + 1) * 16 + j]);
 }
 
-/* One token, H = 2048 (one 32-weight chunk per lane): x arrives already
- * converted (loaded before the routing), so only the weight bytes are
- * waited for once the experts are known.  Same sums as gu_body. */
-template <int RPW>
-DEV void gu_body1(const GUArgs &a, const uint8_t *gbase, const uint8_t *ubase, int r0, const h2 *xl,
-                  const h2 *xh, float Xl, float Xh, _Float16 *out, int lane) {
-    const size_t rb = row_bytes(FQ4K, a.H);
-    Q4Raw g[RPW], u[RPW];
+/* One token, H = 2048 (one 32-weight chunk per lane) of the shared expert: x
+ * arrives already converted (x[0..7] and x[8..15] the chunk's two runs of 16,
+ * Xl and Xh their sums).  Same sums as gu_body. */
+template <int RPW, int SF>
+DEV void gu_body1(const GUArgs &a, const uint8_t *gbase, const uint8_t *ubase, int r0, const h2 *x, float Xl, float Xh,
+                  _Float16 *out, int lane) {
+    const size_t rb = row_bytes(SF, a.H);
+    typename std::conditional<SF == FQ8, Q8Raw, Q4Raw>::type g[RPW], u[RPW];
+    auto load = [&](const uint8_t *row) {
+        if constexpr (SF == FQ8) return q8_load(row, lane);
+        else return q4_load(row, lane);
+    };
+    auto dot = [&](const auto &r) {
+        if constexpr (SF == FQ8) return q8_dot(r, x);
+        else return q4_dot(r, lane, x, x + 8, Xl, Xh);
+    };
 #pragma unroll
     for (int i = 0; i < RPW; i++) {
-        g[i] = q4_load(gbase + (size_t)(r0 + i) * rb, lane);
-        u[i] = q4_load(ubase + (size_t)(r0 + i) * rb, lane);
+        g[i] = load(gbase + (size_t)(r0 + i) * rb);
+        u[i] = load(ubase + (size_t)(r0 + i) * rb);
     }
 #pragma unroll
     for (int i = 0; i < RPW; i++) {
-        const float pg = wave_sum_fast(q4_dot(g[i], lane, xl, xh, Xl, Xh));
-        const float pu = wave_sum_fast(q4_dot(u[i], lane, xl, xh, Xl, Xh));
+        const float pg = wave_sum_fast(dot(g[i])), pu = wave_sum_fast(dot(u[i]));
         if (lane == 0) out[r0 + i] = glu_f16(pg, pu);
     }
 }
@@ -407,22 +416,23 @@ struct PosPack<16> {
  * weights overlap those loads; block 0's waves write the dispatch after
  * their products.  Selection and softmax restate softmax_topk_route
  * (inference/src/shaders.metal:1141-1234) exactly as wave_topk does. */
-template <int EPL>
+template <int EPL, int SF>
 DEV void k_gemv_gate_up1_body(GUArgs a, RouteArgs ra) {
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int rows_blk = 4 * GU_RPW, b = blockIdx.x;
     const int E = a.E, K = a.K;
     int klo;
     q4_pos(lane, klo);
-    if (b >= a.routed_blocks) { /* shared expert (Q4_K): needs no routing */
+    if (b >= a.routed_blocks) { /* shared expert (Q4_K or Q8_0): needs no routing */
+        const int sk = SF == FQ8 ? 32 * lane : klo, sk2 = SF == FQ8 ? 16 : 32; /* this lane's two runs of 16 x */
         f4 xr[8];
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-            xr[q] = *(const f4 *)(a.x + klo + 4 * q);
-            xr[4 + q] = *(const f4 *)(a.x + klo + 32 + 4 * q);
+            xr[q] = *(const f4 *)(a.x + sk + 4 * q);
+            xr[4 + q] = *(const f4 *)(a.x + sk + sk2 + 4 * q);
         }
-        h2 xl[8], xh[8];
-        const float Xl = cvt_x16_f32(xr, xl), Xh = cvt_x16_f32(xr + 4, xh);
+        h2 xs[16];
+        const float Xl = cvt_x16_f32(xr, xs), Xh = cvt_x16_f32(xr + 4, xs + 8);
         const int r0 = (b - a.routed_blocks) * rows_blk + wv * GU_RPW;
         uint32_t sink = 0;
         /* waves 1 and 2 touch the group slots 0..3 of this block's rows (the
@@ -430,7 +440,7 @@ DEV void k_gemv_gate_up1_body(GUArgs a, RouteArgs ra) {
          * H = 2048, S = 512) */
         if ((wv == 1 || wv == 2) && a.pf_sh_down)
             touch_rows8(a.pf_sh_down, a.pf_sh_rb, a.H, b - a.routed_blocks, a.S / rows_blk, 2 * (wv - 1), lane, sink);
-        gu_body1<GU_RPW>(a, a.sh_gate, a.sh_up, r0, xl, xh, Xl, Xh, a.act_sh, lane);
+        gu_body1<GU_RPW, SF>(a, a.sh_gate, a.sh_up, r0, xs, Xl, Xh, a.act_sh, lane);
         asm volatile("s_waitcnt vmcnt(0)" : : "v"(sink));
         return;
     }
@@ -617,7 +627,11 @@ DEV void k_gemv_gate_up1_body(GUArgs a, RouteArgs ra) {
     }
 }
 
-template <int EPL>
+/* SF: the shared expert's format (Q4_K, or the Q8_0 of Q4_K_M files, which
+ * otherwise took the general decode kernel: every wave loading x, the experts
+ * selected block by block: 9.7 us against 6.9 here, one-token layer 18.7 ->
+ * 16.6) */
+template <int EPL, int SF>
 __global__ __launch_bounds__(256) void k_gemv_gate_up1(GUArgs a, RouteArgs ra) {
     /* the arguments the first loads and branches depend on, in one round of
      * scalar loads: left alone, the compiler fetched them in four dependent
@@ -626,7 +640,7 @@ __global__ __launch_bounds__(256) void k_gemv_gate_up1(GUArgs a, RouteArgs ra) {
     asm volatile("" ::"s"(a.kt), "s"(a.routed_blocks), "s"(a.x), "s"(a.gate), "s"(a.up), "s"(a.gate_stride),
                  "s"(a.up_stride), "s"(a.M), "s"(a.E), "s"(a.K), "s"(ra.logits), "s"(ra.bias));
     KT_BEGIN(a.kt);
-    k_gemv_gate_up1_body<EPL>(a, ra);
+    k_gemv_gate_up1_body<EPL, SF>(a, ra);
     KT_END(a.kt);
 }
 
@@ -1304,7 +1318,7 @@ __global__ __launch_bounds__(256) void k_gemv_down_b(DownArgs a) {
 static int epl_of(int E) { return E <= 64 ? 1 : E <= 128 ? 2 : E <= 256 ? 4 : E <= 512 ? 8 : E <= 1024 ? 16 : 0; }
 
 bool gemv_gate_up1_path(int route_in_block, int T, int H, const SharedSide &sh) {
-    return route_in_block && T == 1 && H == 2048 && (!sh.gate || sh.gate_fmt == FQ4K);
+    return route_in_block && T == 1 && H == 2048 && (!sh.gate || sh.gate_fmt == FQ4K || sh.gate_fmt == FQ8);
 }
 
 int launch_gemv_gate_up(const ExpertSide &ex, const SharedSide &sh, const RouteArgs &ra, int route_in_block,
@@ -1316,7 +1330,7 @@ int launch_gemv_gate_up(const ExpertSide &ex, const SharedSide &sh, const RouteA
     if (sh.gate && sh.gate_fmt != FQ4K && sh.gate_fmt != FQ8) return -2;
     GUArgs a;
     a.gate = ex.gate; a.up = ex.up; a.gate_stride = ex.gate_stride; a.up_stride = ex.up_stride;
-    a.sh_gate = sh.gate; a.sh_up = sh.up; a.sh_fmt = sh.gate_fmt; a.S = sh.gate ? sh.S : 0;
+    a.sh_gate = sh.gate; a.sh_up = sh.up; a.sh_fmt = sh.gate ? sh.gate_fmt : FQ4K; a.S = sh.gate ? sh.S : 0;
     a.x = x; a.T = T; a.H = H; a.M = M; a.K = K; a.E = E; a.list = ra.list; a.pairs = ra.pairs;
     a.act = act; a.act_sh = act_sh;
     a.pf_down = a.pf_sh_down = nullptr; a.pf_down_stride = 0; a.pf_rb = a.pf_sh_rb = 0;
@@ -1355,7 +1369,11 @@ int launch_gemv_gate_up(const ExpertSide &ex, const SharedSide &sh, const RouteA
     if (act_by_slot && !gemv_gate_up1_path(route_in_block, T, H, sh)) return -1;
     if (gemv_gate_up1_path(route_in_block, T, H, sh)) {
         a.act_by_slot = act_by_slot;
-#define GU1_LAUNCH(EPLV) KLAUNCH((k_gemv_gate_up1<EPLV>), dim3(blocks), dim3(256), 0, s, a, ra)
+#define GU1_LAUNCH(EPLV)                                                                                   \
+    do {                                                                                                   \
+        if (a.sh_fmt == FQ8) KLAUNCH((k_gemv_gate_up1<EPLV, FQ8>), dim3(blocks), dim3(256), 0, s, a, ra);  \
+        else KLAUNCH((k_gemv_gate_up1<EPLV, FQ4K>), dim3(blocks), dim3(256), 0, s, a, ra);                 \
+    } while (0)
         switch (epl_of(E)) {
             case 1: GU1_LAUNCH(1); break;
             case 2: GU1_LAUNCH(2); break;

@@ -211,6 +211,25 @@ def test_decode_expert_counts(E):
     p.gm.close()
 
 
+@pytest.mark.parametrize("E,kw", [(8, dict(down=13)), (64, {}), (65, dict(M=256, S=512)), (200, dict(down=14)), (256, dict(S=256)),
+                                  (512, {}), (1024, dict(down=13))])
+def test_decode_q8_shared_one_token(E, kw):
+    """The one-token gate/up with a Q8_0 shared expert (its blocks read 34-byte
+    blocks, 32 consecutive inputs a lane) at every width of a lane's expert
+    list, at list edges (65, 200) and with widths that leave the down + combine
+    to the separate kernels: routing and dispatch bit-exact, output within
+    tolerance of the oracle."""
+    banner("decode Q8_0 shared, E=%d %s" % (E, kw))
+    p = Pair(max_tokens=2, E=E, shared=8, seed=170 + E, **kw)
+    for i in range(3):
+        x, h = p.inputs(1, seed=1700 + i)
+        out, dbg = p.run(0, x, h)
+        check_routing(p, x, dbg, 8)
+        ref = p.om.forward(0, x, h)
+        assert rel_l2(out - h, ref - h) < TOL
+    p.gm.close()
+
+
 def test_topk_teacher_forced(base):
     banner("teacher-forced top-k")
     rng = np.random.default_rng(1)
