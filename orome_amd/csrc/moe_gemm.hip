@@ -420,6 +420,14 @@ struct Chunk {
 };
 
 /* ------------------------------------------------------------- tile */
+/* stages per pass of the gate/up loop over a run-time stage count (H other
+ * than 2048; every hidden size taken is a multiple of 4 stages).  The pass
+ * ends in register copies of the weight ring, which wait for its loads, and
+ * a branch around a load or an LDS store makes the wait counts pessimistic:
+ * with two stages a pass and the chunk ends branched, gate/up at T = 300,
+ * H = 3072, E = 128 took 74-78 us, now 64 (61.6 fully unrolled, as H = 2048
+ * is, which is 5 % faster there than this loop); 8 stages a pass: 64. */
+#define GEMM_ROLL 4
 /* One block: Shape<TBM>::W waves, wave w owns RPW row blocks of 16 rows (rows
  * yb*NB + (w*RPW + rb)*16 ..) of NMAT matrices (gate+up, or down).
  * A wave walks units u = (rb, stage j) in order, stage j = 128 k; weight
@@ -465,7 +473,7 @@ DEV void tile_run(const uint8_t *w0, const uint8_t *w1, int in_dim, const _Float
         ch.fetch(src, rowoff, ld, KCH);
         ch.template store<FMT>(xs + Shape<TBM>::XR * BLD);
     }
-    if (nch > 2) ch.fetch(src, rowoff, ld, 2 * KCH);
+    if (nch > 2 || (NST == 0 && RPW == 1)) ch.fetch(src, rowoff, ld, min(2, nch - 1) * KCH);
     __syncthreads();
 
     f4v c[NMAT][TBM];
@@ -474,12 +482,15 @@ DEV void tile_run(const uint8_t *w0, const uint8_t *w1, int in_dim, const _Float
 #pragma unroll
         for (int t = 0; t < TBM; t++) c[m][t] = f4v{0, 0, 0, 0};
 
+    /* LOOP: a stage count only known at run time; ROLL stages per pass */
+    constexpr bool LOOP = NST == 0 && RPW == 1;
+    constexpr int ROLL = LOOP ? GEMM_ROLL : DEPTH;
 #pragma unroll
-    for (int u0 = 0; u0 < U; u0 += DEPTH) {
+    for (int u0 = 0; u0 < U; u0 += ROLL) {
 #pragma unroll
-        for (int d = 0; d < DEPTH; d++) {
-            const int u = u0 + d;
-            const int rb = u / nst, j = u - rb * nst;
+        for (int d0 = 0; d0 < ROLL; d0++) {
+            const int u = u0 + d0, d = d0 % DEPTH;
+            const int rb = RPW == 1 ? 0 : u / nst, j = RPW == 1 ? u : u - rb * nst, odd = RPW == 1 ? d0 & 1 : j & 1;
             /* keep units apart (register pressure): no scheduling across
              * them, and no reuse of B fragments loaded by an earlier unit
              * (row blocks of one wave read the same LDS addresses) */
@@ -489,14 +500,15 @@ DEV void tile_run(const uint8_t *w0, const uint8_t *w1, int in_dim, const _Float
 #pragma unroll
             for (int m = 0; m < NMAT; m++) {
                 cur[m] = ring[d][m];
-                cur[m].prepare(j, kg);
+                cur[m].prepare(odd, kg);
             }
             {
-                const int u2 = min(u + DEPTH, U - 1), rb2 = u2 / nst, j2 = u2 - rb2 * nst;
+                const int u2 = LOOP ? (u + DEPTH < U ? u + DEPTH : u) : min(u + DEPTH, U - 1), rb2 = RPW == 1 ? 0 : u2 / nst,
+                          j2 = LOOP ? (u2 & ~1) + odd : u2 - rb2 * nst;
 #pragma unroll
                 for (int m = 0; m < NMAT; m++) ring[d][m].template load<NT>((m ? rw1 : rw0) + (size_t)rb2 * 16 * rbytes, j2, kg);
             }
-            const _Float16 *bp = xs + ((j >> 1) & 1) * (Shape<TBM>::XR * BLD) + (j & 1) * KC + i * BLD + kg * 8;
+            const _Float16 *bp = xs + ((j >> 1) & 1) * (Shape<TBM>::XR * BLD) + odd * KC + i * BLD + kg * 8;
 #pragma unroll
             for (int s = 0; s < 4; s++) {
                 h8 a[NMAT];
@@ -521,14 +533,23 @@ DEV void tile_run(const uint8_t *w0, const uint8_t *w1, int in_dim, const _Float
                         c[m][t] = mfma(a[m], b[t], c[m][t]);
                     }
             }
-            if (j == nst - 1) {
+            if (!LOOP && j == nst - 1) {
                 epi.template operator()<TBM>(c, rbase + rb * 16 + 4 * kg, tb);
 #pragma unroll
                 for (int m = 0; m < NMAT; m++)
 #pragma unroll
                     for (int t = 0; t < TBM; t++) c[m][t] = f4v{0, 0, 0, 0};
             }
-            if (nch > 2 && (j & 1) && (j >> 1) + 2 < nch) {
+            if (LOOP) {
+                /* no branches around the loads and stores (they would make
+                 * every wait count pessimistic): past the end the last chunk
+                 * comes again, into a buffer that is not read any more */
+                if (odd) {
+                    __syncthreads();
+                    ch.template store<FMT>(xs + ((j >> 1) & 1) * (Shape<TBM>::XR * BLD));
+                    ch.fetch(src, rowoff, ld, min((j >> 1) + 3, nch - 1) * KCH);
+                }
+            } else if (nch > 2 && (j & 1) && (j >> 1) + 2 < nch) {
                 __syncthreads();
                 ch.template store<FMT>(xs + ((j >> 1) & 1) * (Shape<TBM>::XR * BLD));
                 if ((j >> 1) + 3 < nch) ch.fetch(src, rowoff, ld, ((j >> 1) + 3) * KCH);
@@ -537,6 +558,7 @@ DEV void tile_run(const uint8_t *w0, const uint8_t *w1, int in_dim, const _Float
             }
         }
     }
+    if (LOOP) epi.template operator()<TBM>(c, rbase + 4 * kg, tb);
 }
 
 /* Block -> (tile, row block).  Work-groups go to the 8 XCDs round-robin by
@@ -1243,7 +1265,7 @@ int launch_gemm_gate_up(const ExpertSide &ex, const SharedSide &sh, const _Float
         return hipGetLastError() == hipSuccess ? 0 : -3;
     }
     /* compile-time stage count for the common hidden size; other shapes
-     * take the generic loop */
+     * take the loop over a run-time one (GEMM_ROLL) */
 #define GU_LAUNCH(RF, SF, NS)                                                                    \
     do {                                                                                     \
         if (tile_m == GEMM_TILE_SMALL) KLAUNCH((k_gemm_gate_up<RF, SF, NS, GEMM_TILE_SMALL / 16>), grid, block, 0, s, a); \

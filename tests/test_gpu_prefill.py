@@ -520,3 +520,23 @@ def test_two_pass_router_sweep(shape):
             assert np.array_equal(dbg["offsets"], off), "dispatch offsets T=%d" % T
             assert np.array_equal(dbg["pairs"], pairs), "dispatch order T=%d" % T
     p.gm.close()
+
+
+@pytest.mark.parametrize("H,shared", [(512, 12), (1024, 8), (1536, 12), (2560, 8), (3072, 12), (4096, 8)])
+def test_gate_up_stage_counts(H, shared):
+    """The gate/up loop over a run-time stage count (every H but 2048): one
+    pass (H = 512: two activation chunks, both resident), odd numbers of
+    passes and the largest size, on 16- and 32-row tiles (T = 9, 70) and
+    80-row ones (T = 260, K T > 32 E), with a Q4_K and a Q8_0 shared expert.
+    Each equals its unpacked run bit for bit (row-major spans, the same loop)
+    and the oracle within tolerance."""
+    banner("gate/up stage counts, H=%d shared=%d" % (H, shared))
+    p = Pair(max_tokens=260, H=H, E=16, M=256, S=256, shared=shared, seed=H)
+    for T in (9, 70, 260):
+        out, _ = run_and_check(p, T, seed=5000 + T, K=4)
+        x, h = p.inputs(T, seed=5000 + T)
+        p.gm.unpack()
+        plain, _ = p.run(0, x, h, K=4, path=_lib.OROME_PATH_MFMA)
+        p.gm.pack_layers()
+        assert np.array_equal(out, plain), "T=%d" % T
+    p.gm.close()
