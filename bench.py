@@ -269,11 +269,13 @@ def run_config(key, steps, warmup, path, cpu_seconds, no_cpu, graph=True):
     gu_us = stage_us["gate_up"]
     gu_gbs = gu_bytes / (gu_us * 1e-6) / 1e9
     gu_tflops = gu_flops / (gu_us * 1e-6) / 1e12
-    # up to T K = 32 E every expert is in 32-row tiles (one list); above, the
-    # 32-row and 80-row tile lists
+    # up to T K = 32 E every expert is in 32-row tiles (one list), above 44 E
+    # in 80-row tiles, between them in both lists
+    both_lists = 32 * E < T * K <= 44 * E
     kname = {"gemv": "gemv_gate_up", "small_batch_gemm": "gemm_gate_up (16-row tiles)",
              "mfma": ("gemm_gate_up (32-row tile list)" if T * K <= 32 * E
-                      else "gemm_gate_up (32-row + 80-row tile lists)")}[kpath]
+                      else "gemm_gate_up (32-row + 80-row tile lists)" if both_lists
+                      else "gemm_gate_up (80-row tile list)")}[kpath]
     if T >= 2048:
         roof = {"bound": "mfma", "kernel": kname, "achieved": round(gu_tflops, 2),
                 "peak": MFMA_F16_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": round(gu_tflops / MFMA_F16_PEAK_TFLOPS, 4)}
@@ -288,7 +290,7 @@ def run_config(key, steps, warmup, path, cpu_seconds, no_cpu, graph=True):
     if os.path.exists(tf):
         rp = json.load(open(tf))
         traffic = rp.get("gate_up_hbm_bytes_per_launch")
-    serial = kpath == "mfma" and T * K > 32 * E
+    serial = kpath == "mfma" and both_lists
     roof.update({"traffic": traffic, "algorithmic_bytes_per_launch": int(gu_bytes),
                  "algorithmic_flops_per_launch": gu_flops, "avg_launch_us": gu_us,
                  "timing": "HIP events recorded by the gate/up launches themselves (hipExtLaunchKernel "

@@ -696,9 +696,8 @@ static int forward_impl(orome_hip_ctx *c, const OromeHipModelConfig *cfg, const 
             TLAUNCH(c, ST_DISPATCH, launch_dispatch(a, c->tiles, c->tiles_b, S ? 1 : 0, c->dcount, s, a.dcnt ? 1 : 0), "dispatch");
         const GemmSelfDispatch sdargs = {c->dcount, dispatch_blocks(T), c->tmask, c->idx, c->offsets, c->pairs, c->pos};
         /* one launch per tile list (grid sized for the most tiles it can hold) */
-        /* small batches (T K <= 32 E): every expert in 32-row tiles, the
-         * shared expert too, and no big-tile list */
-        const bool sh_small = (long)T * K <= (long)GEMM_TILE_SMALL * E;
+        const int lists = gemm_lists(T, K, E);
+        const bool sh_small = lists == LISTS_SMALL;
         const int ns_max = E + (sh_small ? (T * K) / GEMM_TILE_SMALL : 0) +
                            (S && sh_small ? (T + GEMM_TILE_SMALL - 1) / GEMM_TILE_SMALL : 0),
                   nb_max = (T * K) / GEMM_TILE_BIG + E + (S && !sh_small ? (T + GEMM_TILE_BIG - 1) / GEMM_TILE_BIG : 0);
@@ -721,9 +720,10 @@ static int forward_impl(orome_hip_ctx *c, const OromeHipModelConfig *cfg, const 
                        : launch_gemm_down(exm, shm, c->act, c->act_sh, c->tmax * c->kmax, c->tmax, T, H, M, K, E, tm, c->tiles_b, nb_max, c->y,
                                           c->ysh, st);
         };
-        if (sh_small) { /* one list */
-            TLAUNCH(c, ST_GATE_UP, gate_up(GEMM_TILE_SMALL, s), "grouped gate/up");
-            TLAUNCH(c, ST_DOWN, down(GEMM_TILE_SMALL, s), "grouped down");
+        if (lists != LISTS_BOTH) { /* one list */
+            const int tm = sh_small ? GEMM_TILE_SMALL : GEMM_TILE_BIG;
+            TLAUNCH(c, ST_GATE_UP, gate_up(tm, s), "grouped gate/up");
+            TLAUNCH(c, ST_DOWN, down(tm, s), "grouped down");
         } else if (c->timing || !c->side) { /* per-stage timing (or no side stream): both lists in order on one stream */
             TLAUNCH(c, ST_GATE_UP, (gate_up(GEMM_TILE_SMALL, s) ? -3 : gate_up(GEMM_TILE_BIG, s)), "grouped gate/up");
             TLAUNCH(c, ST_DOWN, (down(GEMM_TILE_SMALL, s) ? -3 : down(GEMM_TILE_BIG, s)), "grouped down");

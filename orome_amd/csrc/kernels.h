@@ -201,11 +201,23 @@ int launch_fill_u32(void *p, uint32_t v, size_t words, hipStream_t s);
 
 /* tile list for the grouped GEMM: tiles[0] = count, then (expert, first, rows)
  * triples; expert == E denotes the shared expert over all T tokens */
-/* two tile lists per call: experts with <= GEMM_TILE_SMALL rows (one small
- * tile each) and the rest in tiles of GEMM_TILE_BIG rows; while T*K <=
- * GEMM_TILE_SMALL*E every expert is cut into small tiles and the shared
- * expert joins the small list (the big list is empty).  Capacities: small
- * 2E + T/SMALL + 1, big T*K/BIG + E + T/BIG + 1. */
+/* The lists of a call (gemm_lists):
+ *   LISTS_SMALL (T*K <= 32 E)  every expert cut into tiles of GEMM_TILE_SMALL
+ *                 rows, the shared expert in the same list;
+ *   LISTS_BOTH    experts with <= GEMM_TILE_SMALL rows one small tile each,
+ *                 the rest and the shared expert tiles of GEMM_TILE_BIG, the
+ *                 big list on a second stream beside the small one;
+ *   LISTS_BIG (T*K > GEMM_BIG_ONLY E)  every expert in tiles of
+ *                 GEMM_TILE_BIG: the few small experts cost less there than a
+ *                 nearly empty pair of launches and the two streams' fork and
+ *                 join (~20 us a layer launched eagerly).  Layers of 256
+ *                 experts, K = 8, both lists -> big only: T = 2048 317 -> 293
+ *                 us, 1500 293 -> 271, 4096 613 -> 591; 1300 (40 rows an
+ *                 expert) 765 -> 766 for three layers; 1100 (34 rows) 239 ->
+ *                 250.
+ * Capacities: small 2E + T/SMALL + 1, big T*K/BIG + E + T/BIG + 1. */
+enum { LISTS_SMALL, LISTS_BOTH, LISTS_BIG };
+#define GEMM_BIG_ONLY 44
 #define GEMM_TILE_SMALL 32
 /* 16-row tiles for lists whose experts hold at most 16 rows (the small-batch
  * path: T <= 16); per-tile kernels only */
@@ -213,3 +225,7 @@ int launch_fill_u32(void *p, uint32_t v, size_t words, hipStream_t s);
 #ifndef GEMM_TILE_BIG
 #define GEMM_TILE_BIG 80
 #endif
+static inline __host__ __device__ int gemm_lists(int T, int K, int E) {
+    const long tk = (long)T * K;
+    return tk <= (long)GEMM_TILE_SMALL * E ? LISTS_SMALL : tk > (long)GEMM_BIG_ONLY * E ? LISTS_BIG : LISTS_BOTH;
+}

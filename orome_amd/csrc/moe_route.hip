@@ -536,11 +536,10 @@ __global__ __launch_bounds__(256) void k_topk_exact(RouteArgs a) {
  *  2. scan:    one block: per expert an exclusive scan of cnt over blocks
  *              (in place) and the total; block scans of the totals give the
  *              offsets, active-expert ranks and GEMM tile offsets; then the
- *              active list and two GEMM tile lists (expert, first row, rows):
- *              experts with <= GEMM_TILE_SMALL rows get one small tile, the
- *              others tiles of GEMM_TILE_BIG rows; the shared expert (id E)
- *              covers tokens 0..T-1 in small tiles when the average expert
- *              has <= GEMM_TILE_SMALL rows, else in big ones.
+ *              active list and the GEMM tile lists (expert, first row, rows)
+ *              of gemm_lists; the shared expert (id E) covers tokens 0..T-1
+ *              in small tiles when the average expert has <=
+ *              GEMM_TILE_SMALL rows, else in big ones.
  *  3. scatter: per block, the same masks; a pair's rank is its expert's
  *              offset + the block's base + the popcount of the mask below
  *              its token. */
@@ -579,18 +578,16 @@ __global__ __launch_bounds__(DSP_TOK) void k_dispatch_count(RouteArgs a, uint32_
     }
 }
 
-/* Tiles of one expert: rows <= GEMM_TILE_SMALL -> one small tile, else
- * ceil(rows / GEMM_TILE_BIG) big tiles.  While the batch is small (T K <=
- * GEMM_TILE_SMALL E, tile_small_only) every expert is cut into small tiles:
- * the few big experts of a skewed routing would otherwise leave most CUs
- * idle in a big-tile launch of their own, and the shared expert is in the
- * small list then anyway (the host launches only that list). */
-DEV bool tile_small_only(const RouteArgs &a) { return (size_t)a.T * a.K <= (size_t)GEMM_TILE_SMALL * a.E; }
-DEV uint32_t n_small_tiles(uint32_t c, bool so) {
-    return so ? (c + GEMM_TILE_SMALL - 1) / GEMM_TILE_SMALL : c != 0 && c <= GEMM_TILE_SMALL;
+/* Tiles of one expert in the call's lists (gemm_lists).  While the batch is
+ * small every expert is cut into small tiles: the few big experts of a
+ * skewed routing would otherwise leave most CUs idle in a big-tile launch of
+ * their own. */
+DEV uint32_t n_small_tiles(uint32_t c, int lists) {
+    return lists == LISTS_SMALL ? (c + GEMM_TILE_SMALL - 1) / GEMM_TILE_SMALL
+                                : lists == LISTS_BOTH && c != 0 && c <= GEMM_TILE_SMALL;
 }
-DEV uint32_t n_big_tiles(uint32_t c, bool so) {
-    return !so && c > GEMM_TILE_SMALL ? (c + GEMM_TILE_BIG - 1) / GEMM_TILE_BIG : 0;
+DEV uint32_t n_big_tiles(uint32_t c, int lists) {
+    return lists == LISTS_BIG || (lists == LISTS_BOTH && c > GEMM_TILE_SMALL) ? (c + GEMM_TILE_BIG - 1) / GEMM_TILE_BIG : 0;
 }
 DEV void put_tiles(uint32_t *list, uint32_t t0, uint32_t e, uint32_t first, uint32_t c, uint32_t tm) {
     for (uint32_t j = 0; j * tm < c; j++) {
@@ -611,9 +608,10 @@ DEV void dispatch_lists(const RouteArgs &a, uint32_t c, uint32_t *xo, uint32_t *
     /* glob false: the exclusive offsets into xo only (the blocks of a
      * dispatch that one other block writes the lists for) */
     const int E = a.E, T = a.T, tid = threadIdx.x;
-    const bool so = tile_small_only(a), mine = tid < E;
+    const int lists = gemm_lists(T, a.K, E);
+    const bool so = lists == LISTS_SMALL, mine = tid < E;
     if (!mine) c = 0;
-    const uint32_t ns_own = n_small_tiles(c, so), nb_own = n_big_tiles(c, so);
+    const uint32_t ns_own = n_small_tiles(c, lists), nb_own = n_big_tiles(c, lists);
     uint32_t x = c | ((uint32_t)(c != 0) << 16), y = ns_own | (nb_own << 16), tx, ty;
     scan2_block(x, y, wsum, tx, ty);
     if (mine) {
@@ -628,7 +626,7 @@ DEV void dispatch_lists(const RouteArgs &a, uint32_t c, uint32_t *xo, uint32_t *
             const uint32_t r = (x >> 16) - 1;
             ACT_E(a.list, r) = (uint32_t)tid;
             ACT_OFF(a.list, E, r) = o;
-            if (c <= GEMM_TILE_SMALL || so)
+            if (ns_own)
                 put_tiles(tiles_s, (y & 0xFFFFu) - ns_own, (uint32_t)tid, o, c, GEMM_TILE_SMALL);
             else put_tiles(tiles_b, (y >> 16) - nb_own, (uint32_t)tid, o, c, GEMM_TILE_BIG);
         }

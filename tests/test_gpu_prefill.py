@@ -540,3 +540,22 @@ def test_gate_up_stage_counts(H, shared):
         p.gm.pack_layers()
         assert np.array_equal(out, plain), "T=%d" % T
     p.gm.close()
+
+
+@pytest.mark.parametrize("T", [128, 129, 176, 177, 300])
+@pytest.mark.parametrize("kw", [dict(), dict(zipf=True, down=14), dict(S=0, zipf=True), dict(shared=8, down=13)])
+def test_tile_lists_at_their_limits(T, kw):
+    """Both sides of the limits between the call's tile lists (16 experts, K =
+    4: 32-row tiles up to T = 128, both lists up to 176, 80-row tiles alone
+    above), with skewed routing (experts of no, one and many rows in every
+    list), without a shared expert, and with routed and shared formats that
+    take separate walks: routing and dispatch bit-exact, output within
+    tolerance of the oracle, unpacked run bit for bit."""
+    banner("tile lists T=%d %s" % (T, kw))
+    p = Pair(max_tokens=300, **{**dict(H=2048, E=16, M=512, S=512, seed=90), **kw})
+    out, _ = run_and_check(p, T, seed=6000 + T, K=4)
+    x, h = p.inputs(T, seed=6000 + T)
+    p.gm.unpack()
+    plain, _ = p.run(0, x, h, K=4, path=_lib.OROME_PATH_MFMA)
+    assert np.array_equal(out, plain)
+    p.gm.close()
