@@ -580,6 +580,8 @@ struct GemmArgs {
     int zrow, zrow_sh;        /* all-zero rows of src / src_sh (rows past a tile read them) */
     int nyb;                  /* row blocks per tile */
     int uwin;                 /* tiles walked: all (0), the last uwin (> 0) or all but the last -uwin (< 0) */
+    int urev;                 /* units dealt to an XCD's blocks from the last one down (a second walk) */
+    int fmt, fmt_sh;          /* two walks: formats of the routed and the shared matrices */
     const uint32_t *tiles, *pairs;
     _Float16 *act, *act_sh;   /* gate/up outputs */
     unsigned long long *kt;   /* gate/up: per-block launch stamps (KT_BEGIN / KT_END) or NULL */
@@ -757,8 +759,9 @@ struct UnitDesc {
  * blocks of that XCD (work-groups are dealt to the 8 XCDs round-robin by
  * linear id), so the row blocks of one tile share an L2 and run at about the
  * same time; within an XCD, block `slot` takes units slot, slot + bpx, ... */
-DEV UnitDesc unit_desc(const uint32_t *tiles, int nyb, int E, int n, int uwin) {
-    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, bpx = gridDim.x >> 3;
+DEV UnitDesc unit_desc(const uint32_t *tiles, int nyb, int E, int n, int uwin, int urev) {
+    const int xcd = blockIdx.x & 7, bpx = gridDim.x >> 3, bslot = (int)(blockIdx.x >> 3);
+    const int slot = urev ? bpx - 1 - bslot : bslot;
     const int q = slot + n * bpx, ti = 8 * (q / nyb) + xcd;
     /* the list is read-only here: constant address space, so the uniform
      * reads are scalar loads and do not wait behind the weight loads */
@@ -956,7 +959,7 @@ struct GuPol {
     const GemmArgs &a;
     MDEV int in_dim() const { return a.H; }
     MDEV int ld() const { return a.H; }
-    MDEV UnitDesc desc(int n) const { return unit_desc(a.tiles, a.nyb, a.E, n, a.uwin); }
+    MDEV UnitDesc desc(int n) const { return unit_desc(a.tiles, a.nyb, a.E, n, a.uwin, a.urev); }
     MDEV const _Float16 *src(const UnitDesc &) const { return a.src; }
     MDEV const uint8_t *weights(const UnitDesc &u, int m) const {
         return u.sh ? (m ? a.sh_b : a.sh_a) : m ? a.wb + (size_t)u.e * a.stride_b : a.wa + (size_t)u.e * a.stride_a;
@@ -980,7 +983,7 @@ struct DnPol {
     const GemmArgs &a;
     MDEV int in_dim() const { return a.M; }
     MDEV int ld() const { return a.M; }
-    MDEV UnitDesc desc(int n) const { return unit_desc(a.tiles, a.nyb, a.E, n, a.uwin); }
+    MDEV UnitDesc desc(int n) const { return unit_desc(a.tiles, a.nyb, a.E, n, a.uwin, a.urev); }
     MDEV const _Float16 *src(const UnitDesc &u) const { return u.sh ? a.src_sh : a.src; }
     MDEV const uint8_t *weights(const UnitDesc &u, int) const { return u.sh ? a.sh_a : a.wa + (size_t)u.e * a.stride_a; }
     MDEV uint32_t row_raw(const UnitDesc &u, int q) const { return !u.valid || q >= u.rows ? ~0u : (uint32_t)(u.first + q); }
@@ -1127,6 +1130,55 @@ __global__ __launch_bounds__(Shape<TBM>::W * 64) void k_gemm_down_p(GemmArgs a) 
     tile_stream<EFMT, 1, DN_RPW, Shape<TBM>::DEPTH, 4, TBM>(DnPol{a}, xs, rowoff);
 }
 
+/* Routed and shared matrices of two tile-major formats in one launch: a
+ * block walks its routed units, then its units of the shared expert's tiles
+ * (they end the list), which are dealt from the other end of each XCD's
+ * blocks, first to those that had a routed unit less.  As two launches the
+ * second one's few units ran alone, about one a CU, behind the first one's
+ * last round: 4096 tokens with a Q6_K down and a Q4_K shared one 572 -> 561 us
+ * a layer, 777 with Q5_K and a Q8_0 shared expert 185 -> 181, 512 with skewed
+ * routing and a Q6_K down 125 -> 122.5.  (Row-major formats keep a launch
+ * each: their walks take more registers than one kernel has for both.) */
+DEV void two_walks(const GemmArgs &a, GemmArgs &ar, GemmArgs &as) {
+    ar = a;
+    as = a;
+    ar.uwin = -a.nsh;
+    as.uwin = a.nsh;
+    as.urev = 1;
+}
+template <int TBM>
+__global__ __launch_bounds__(Shape<TBM>::W * 64) void k_gemm_down_p2(GemmArgs a) {
+    GEMM_PIN_ARGS(a, "s"(a.y), "s"(a.ysh), "s"(a.nsh), "s"(a.fmt), "s"(a.fmt_sh));
+    static_assert(TBM >= 2, "persistent kernels take 32- and 80-row tiles");
+    __shared__ __attribute__((aligned(16))) _Float16 xs[3 * Shape<TBM>::XR * BLD];
+    __shared__ int rowoff[3 * TBM * 16];
+    GemmArgs ar, as;
+    two_walks(a, ar, as);
+#define WALK(F, ARGS) tile_stream<F, 1, DN_RPW, Shape<TBM>::DEPTH, 4, TBM>(DnPol{ARGS}, xs, rowoff)
+    if (a.fmt == FQ4KT) WALK(FQ4KT, ar);
+    else if (a.fmt == FQ5KT) WALK(FQ5KT, ar);
+    else WALK(FQ6KT, ar); /* (the launcher sends no other routed format) */
+    __syncthreads();
+    if (a.fmt_sh == FQ4KT) WALK(FQ4KT, as);
+    else if (a.fmt_sh == FQ5KT) WALK(FQ5KT, as);
+    else if (a.fmt_sh == FQ6KT) WALK(FQ6KT, as);
+    else WALK(FQ8T, as);
+#undef WALK
+}
+template <int TBM>
+__global__ __launch_bounds__(Shape<TBM>::W * 64) void k_gemm_gate_up_p2(GemmArgs a) {
+    GEMM_PIN_ARGS(a, "s"(a.act), "s"(a.act_sh), "s"(a.nsh));
+    __shared__ __attribute__((aligned(16))) _Float16 xs[3 * Shape<TBM>::XR * BLD];
+    __shared__ int rowoff[3 * TBM * 16];
+    KT_BEGIN(a.kt);
+    GemmArgs ar, as;
+    two_walks(a, ar, as);
+    tile_stream<FQ4KT, 2, GU_RPW, Shape<TBM>::DEPTH, 16, TBM>(GuPol{ar}, xs, rowoff);
+    __syncthreads();
+    tile_stream<FQ8T, 2, GU_RPW, 2, 16, TBM>(GuPol{as}, xs, rowoff);
+    KT_END(a.kt);
+}
+
 /* Persistent grid: one block per CU, a multiple of the 8 XCDs.  The
  * environment variable OROME_GEMM_PERSIST_BLOCKS overrides it (tests use a
  * small grid to give every block many units); 0 selects the per-tile
@@ -1247,7 +1299,10 @@ int launch_gemm_gate_up(const ExpertSide &ex, const SharedSide &sh, const _Float
         else KLAUNCH((k_gemm_gate_up_p<GEMM_TILE_SMALL / 16, GF>), dim3(pb), block, 0, s, ARGS);          \
     } while (0)
         const int nsh = shared_tiles_in(sh, T, K, E, tile_m);
-        if (nsh && q8) { /* Q8_0 shared expert: one walk over the routed tiles, one over the shared */
+        if (nsh && tiled && sh.gate_fmt == FQ8T && tile_m == GEMM_TILE_BIG) { /* Q8_0 shared expert: two walks */
+            a.nsh = nsh;
+            KLAUNCH((k_gemm_gate_up_p2<GEMM_TILE_BIG / 16>), dim3(pb), block, 0, s, a);
+        } else if (nsh && q8) { /* (a launch for the routed tiles, one for the shared) */
             GemmArgs ar = a, as = a;
             ar.uwin = -nsh;
             as.uwin = nsh;
@@ -1325,7 +1380,13 @@ int launch_gemm_down(const ExpertSide &ex, const SharedSide &sh, const _Float16 
     } while (0)
         if (!mixed) {
             DP_TILE(ex.down_fmt, a);
-        } else { /* routed and shared down differ in format: one walk each */
+        } else if (TILED(ex.down_fmt) && ex.down_fmt != FQ8T) { /* routed and shared down differ in format: two walks */
+            a.nsh = nsh;
+            a.fmt = ex.down_fmt;
+            a.fmt_sh = sf;
+            if (tile_m == GEMM_TILE_BIG) KLAUNCH((k_gemm_down_p2<GEMM_TILE_BIG / 16>), dim3(pb), block, 0, s, a);
+            else KLAUNCH((k_gemm_down_p2<GEMM_TILE_SMALL / 16>), dim3(pb), block, 0, s, a);
+        } else { /* (a launch each) */
             GemmArgs ar = a, as = a;
             ar.uwin = -nsh;
             as.uwin = nsh;

@@ -559,3 +559,19 @@ def test_tile_lists_at_their_limits(T, kw):
     plain, _ = p.run(0, x, h, K=4, path=_lib.OROME_PATH_MFMA)
     assert np.array_equal(out, plain)
     p.gm.close()
+
+
+@pytest.mark.parametrize("T", [129, 177, 300])
+@pytest.mark.parametrize("down,shared,shared_down", [(12, 8, 8), (12, 12, 13), (13, 8, 12), (13, 12, 14), (14, 12, 13), (14, 8, 8)])
+def test_routed_and_shared_formats_in_one_launch(T, down, shared, shared_down):
+    """Q4_K / Q5_K / Q6_K routed down matrices beside a shared expert in
+    another format: the packed layer walks both in one launch and has to equal,
+    bit for bit, the unpacked one (a launch each)."""
+    banner("two walks T=%d %d %d %d" % (T, down, shared, shared_down))
+    p = Pair(max_tokens=300, H=2048, E=16, M=512, S=512, seed=91, down=down, shared=shared, shared_down=shared_down)
+    out, _ = run_and_check(p, T, seed=6100 + T, K=4)
+    x, h = p.inputs(T, seed=6100 + T)
+    p.gm.unpack()
+    plain, _ = p.run(0, x, h, K=4, path=_lib.OROME_PATH_MFMA)
+    assert np.array_equal(out, plain)
+    p.gm.close()
