@@ -1135,10 +1135,11 @@ __global__ __launch_bounds__(Shape<TBM>::W * 64) void k_gemm_down_p(GemmArgs a) 
  * (they end the list), which are dealt from the other end of each XCD's
  * blocks, first to those that had a routed unit less.  As two launches the
  * second one's few units ran alone, about one a CU, behind the first one's
- * last round: 4096 tokens with a Q6_K down and a Q4_K shared one 572 -> 561 us
- * a layer, 777 with Q5_K and a Q8_0 shared expert 185 -> 181, 512 with skewed
- * routing and a Q6_K down 125 -> 122.5.  (Row-major formats keep a launch
- * each: their walks take more registers than one kernel has for both.) */
+ * last round.  Layer speed against one earlier build, two launches -> one:
+ * 4096 tokens with a Q6_K down and a Q4_K shared one 1.044 -> 1.066 (about
+ * 12 us of 572), 777 tokens with Q5_K and a Q8_0 shared expert 1.002 ->
+ * 1.023, 512 with skewed routing and a Q6_K down 1.003 -> 1.027.  (Row-major
+ * layers keep a launch each: their Q8_0 walk spills registers by itself.) */
 DEV void two_walks(const GemmArgs &a, GemmArgs &ar, GemmArgs &as) {
     ar = a;
     as = a;
