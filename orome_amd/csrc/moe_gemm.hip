@@ -421,12 +421,17 @@ struct Chunk {
 
 /* ------------------------------------------------------------- tile */
 /* stages per pass of the gate/up loop over a run-time stage count (H other
- * than 2048; every hidden size taken is a multiple of 4 stages).  The pass
- * ends in register copies of the weight ring, which wait for its loads, and
- * a branch around a load or an LDS store makes the wait counts pessimistic:
- * with two stages a pass and the chunk ends branched, gate/up at T = 300,
- * H = 3072, E = 128 took 74-78 us, now 64 (61.6 fully unrolled, as H = 2048
- * is, which is 5 % faster there than this loop); 8 stages a pass: 64. */
+ * than 2048; every hidden size taken is a multiple of GEMM_ROLL stages).  The
+ * pass ends in register copies of the weight ring, which wait for its loads,
+ * and a branch around a load or an LDS store makes the wait counts
+ * pessimistic: with two stages a pass and the chunk ends branched, gate/up at
+ * T = 300, H = 3072, E = 128 took 74-78 us, now 64 (61.6 fully unrolled, as
+ * H = 2048 is, which is 5 % faster there than this loop); 8 stages a pass:
+ * 64.  Row-major Q8_0 (eight 2-byte aligned loads a stage and matrix) keeps
+ * the branched form, a ring's length a pass: four stages a pass took its
+ * 32-row kernel to 242 + 24 registers (one wave a SIMD) and made the 80-row
+ * one spill.  Layers with such a shared expert, four stages -> this: 37
+ * tokens 186.5 -> 173.6 us, 5 tokens at H = 3072 117 -> 102, 512 254 -> 245. */
 #define GEMM_ROLL 4
 /* One block: Shape<TBM>::W waves, wave w owns RPW row blocks of 16 rows (rows
  * yb*NB + (w*RPW + rb)*16 ..) of NMAT matrices (gate+up, or down).
@@ -446,6 +451,8 @@ DEV void tile_run(const uint8_t *w0, const uint8_t *w1, int in_dim, const _Float
      * completely and the prefetch ring never crosses a loop back-edge (where
      * the register copies would wait for every load in flight) */
     const int nst = NST ? NST : in_dim / KC, nch = nst / 2, U = RPW * nst;
+    /* LOOP: a stage count only known at run time, GEMM_ROLL stages per pass */
+    constexpr bool LOOP = NST == 0 && RPW == 1 && FMT != FQ8;
     const int rbase = yb * (Shape<TBM>::W * 16 * RPW) + wv * 16 * RPW;
     const uint8_t *rw0 = w0 + lane_row<FMT>(rbase, i, rbytes);
     const uint8_t *rw1 = NMAT > 1 ? w1 + lane_row<FMT>(rbase, i, rbytes) : nullptr;
@@ -473,7 +480,7 @@ DEV void tile_run(const uint8_t *w0, const uint8_t *w1, int in_dim, const _Float
         ch.fetch(src, rowoff, ld, KCH);
         ch.template store<FMT>(xs + Shape<TBM>::XR * BLD);
     }
-    if (nch > 2 || (NST == 0 && RPW == 1)) ch.fetch(src, rowoff, ld, min(2, nch - 1) * KCH);
+    if (nch > 2 || LOOP) ch.fetch(src, rowoff, ld, min(2, nch - 1) * KCH);
     __syncthreads();
 
     f4v c[NMAT][TBM];
@@ -482,9 +489,8 @@ DEV void tile_run(const uint8_t *w0, const uint8_t *w1, int in_dim, const _Float
 #pragma unroll
         for (int t = 0; t < TBM; t++) c[m][t] = f4v{0, 0, 0, 0};
 
-    /* LOOP: a stage count only known at run time; ROLL stages per pass */
-    constexpr bool LOOP = NST == 0 && RPW == 1;
     constexpr int ROLL = LOOP ? GEMM_ROLL : DEPTH;
+    static_assert(ROLL % DEPTH == 0 && (RPW != 1 || ROLL % 2 == 0), "a pass refills the whole ring and ends chunks at odd stages");
 #pragma unroll
     for (int u0 = 0; u0 < U; u0 += ROLL) {
 #pragma unroll
@@ -1210,7 +1216,8 @@ static int tile_waves(int tile_m) {
 static int gate_up_shape(const ExpertSide &ex, const SharedSide &sh, int H, int M, int tile_m) {
     const int W = tile_waves(tile_m);
     const int NB = W * 16 * GU_RPW;
-    if ((H / KC * GU_RPW) % 4) return -2; /* every ring depth used divides the unit count */
+    static_assert(GEMM_ROLL % Shape<GEMM_TILE_SMALL / 16>::DEPTH == 0 && GEMM_ROLL % Shape<GEMM_TILE_BIG / 16>::DEPTH == 0, "ring depths");
+    if ((H / KC * GU_RPW) % GEMM_ROLL) return -2; /* every pass and ring depth used divides the unit count */
     if (H % KCH || M % NB || (sh.gate && sh.S % NB) || (ex.gate_fmt != FQ4K && ex.gate_fmt != FQ4KT)) return -2;
     /* shared expert: the routed format, or Q8_0 (row-major, or tile-major
      * beside tile-major routed matrices) */

@@ -3,6 +3,7 @@ against an independent reader, error paths, and the synthetic generator."""
 import ctypes as C
 import os
 import re
+import struct
 import subprocess
 
 import numpy as np
@@ -181,3 +182,40 @@ def test_synth_centered_q4k_mins_equal_scales():
         assert float(b[2:4].view(np.float16)[0]) == float(np.float16(7.5 * d))
     w = O.decode_rows(O.Q4_K, om.array("blk.0.ffn_gate_exps.weight")[:144 * 8 * 512], 512, 2048)
     assert abs(w.mean()) < 0.02 * w.std()
+
+
+def kernel_descriptors():
+    """(scratch bytes a lane, registers a lane) of every kernel in the built
+    library: the kernel descriptors (symbols NAME.kd) of its code objects."""
+    blob, out = open(_lib.LIB_PATH, "rb").read(), {}
+    magic = b"__CLANG_OFFLOAD_BUNDLE__"
+    for m in re.finditer(magic, blob):
+        at = m.end() + 8
+        for _ in range(struct.unpack_from("<Q", blob, m.end())[0]):
+            off, size, n = struct.unpack_from("<QQQ", blob, at)
+            at += 24 + n
+            elf = blob[m.start() + off:m.start() + off + size]
+            if b"gfx950" not in blob[at - n:at] or elf[:4] != b"\x7fELF":
+                continue
+            shoff, = struct.unpack_from("<Q", elf, 40)
+            shsize, shnum = struct.unpack_from("<HH", elf, 58)
+            secs = [struct.unpack_from("<IIQQQQIIQQ", elf, shoff + k * shsize) for k in range(shnum)]
+            for sec in (s for s in secs if s[1] == 2):  # symbol table
+                strings = secs[sec[6]][4]
+                for k in range(sec[4], sec[4] + sec[5], 24):
+                    name, _, _, ndx, value, _ = struct.unpack_from("<IBBHQQ", elf, k)
+                    name = elf[strings + name:elf.index(b"\0", strings + name)].decode()
+                    if name.endswith(".kd"):
+                        kd = value - secs[ndx][3] + secs[ndx][4]
+                        scratch, rsrc1 = struct.unpack_from("<I", elf, kd + 4)[0], struct.unpack_from("<I", elf, kd + 48)[0]
+                        out[name[:-3]] = scratch, 8 * ((rsrc1 & 63) + 1)
+    return out
+
+
+def test_tile_gate_up_kernels_keep_their_registers():
+    """The per-tile gate/up kernels, whose routed and shared loops share one
+    register allocation, spill nothing and leave room for two waves on each
+    SIMD (512 registers a lane), whatever the shared expert's format."""
+    ks = {k: v for k, v in kernel_descriptors().items() if re.match(r"_Z\d+k_gemm_gate_upI", k)}
+    assert len(ks) >= 20
+    assert not {k: v for k, v in ks.items() if v[0] or v[1] > 256}
