@@ -586,7 +586,6 @@ struct GemmArgs {
     int zrow, zrow_sh;        /* all-zero rows of src / src_sh (rows past a tile read them) */
     int nyb;                  /* row blocks per tile */
     int uwin;                 /* tiles walked: all (0), the last uwin (> 0) or all but the last -uwin (< 0) */
-    int urev;                 /* units dealt to an XCD's blocks from the last one down (a second walk) */
     int fmt, fmt_sh;          /* two walks: formats of the routed and the shared matrices */
     const uint32_t *tiles, *pairs;
     _Float16 *act, *act_sh;   /* gate/up outputs */
@@ -764,10 +763,12 @@ struct UnitDesc {
 /* The n-th unit of this block.  Units of tiles t = xcd (mod 8) go to the
  * blocks of that XCD (work-groups are dealt to the 8 XCDs round-robin by
  * linear id), so the row blocks of one tile share an L2 and run at about the
- * same time; within an XCD, block `slot` takes units slot, slot + bpx, ... */
-DEV UnitDesc unit_desc(const uint32_t *tiles, int nyb, int E, int n, int uwin, int urev) {
+ * same time; within an XCD, block `slot` takes units slot, slot + bpx, ...
+ * REV: the XCD's last block is slot 0 (a second walk). */
+template <bool REV>
+DEV UnitDesc unit_desc(const uint32_t *tiles, int nyb, int E, int n, int uwin) {
     const int xcd = blockIdx.x & 7, bpx = gridDim.x >> 3, bslot = (int)(blockIdx.x >> 3);
-    const int slot = urev ? bpx - 1 - bslot : bslot;
+    const int slot = REV ? bpx - 1 - bslot : bslot;
     const int q = slot + n * bpx, ti = 8 * (q / nyb) + xcd;
     /* the list is read-only here: constant address space, so the uniform
      * reads are scalar loads and do not wait behind the weight loads */
@@ -961,11 +962,12 @@ DEV void tile_stream(const P &pol, _Float16 *xs, int *rowoff) {
     }
 }
 
+template <bool REV = false>
 struct GuPol {
     const GemmArgs &a;
     MDEV int in_dim() const { return a.H; }
     MDEV int ld() const { return a.H; }
-    MDEV UnitDesc desc(int n) const { return unit_desc(a.tiles, a.nyb, a.E, n, a.uwin, a.urev); }
+    MDEV UnitDesc desc(int n) const { return unit_desc<REV>(a.tiles, a.nyb, a.E, n, a.uwin); }
     MDEV const _Float16 *src(const UnitDesc &) const { return a.src; }
     MDEV const uint8_t *weights(const UnitDesc &u, int m) const {
         return u.sh ? (m ? a.sh_b : a.sh_a) : m ? a.wb + (size_t)u.e * a.stride_b : a.wa + (size_t)u.e * a.stride_a;
@@ -985,11 +987,12 @@ struct GuPol {
     }
 };
 
+template <bool REV = false>
 struct DnPol {
     const GemmArgs &a;
     MDEV int in_dim() const { return a.M; }
     MDEV int ld() const { return a.M; }
-    MDEV UnitDesc desc(int n) const { return unit_desc(a.tiles, a.nyb, a.E, n, a.uwin, a.urev); }
+    MDEV UnitDesc desc(int n) const { return unit_desc<REV>(a.tiles, a.nyb, a.E, n, a.uwin); }
     MDEV const _Float16 *src(const UnitDesc &u) const { return u.sh ? a.src_sh : a.src; }
     MDEV const uint8_t *weights(const UnitDesc &u, int) const { return u.sh ? a.sh_a : a.wa + (size_t)u.e * a.stride_a; }
     MDEV uint32_t row_raw(const UnitDesc &u, int q) const { return !u.valid || q >= u.rows ? ~0u : (uint32_t)(u.first + q); }
@@ -1115,7 +1118,7 @@ DEV void k_gemm_gate_up_p_body(GemmArgs a) {
     static_assert(TBM >= 2, "persistent kernels take 32- and 80-row tiles");
     __shared__ __attribute__((aligned(16))) _Float16 xs[3 * Shape<TBM>::XR * BLD];
     __shared__ int rowoff[3 * TBM * 16];
-    tile_stream<GF, 2, GU_RPW, (GF == FQ8 || GF == FQ8T ? 2 : Shape<TBM>::DEPTH), 16, TBM>(GuPol{a}, xs, rowoff);
+    tile_stream<GF, 2, GU_RPW, (GF == FQ8 || GF == FQ8T ? 2 : Shape<TBM>::DEPTH), 16, TBM>(GuPol<>{a}, xs, rowoff);
 }
 
 template <int TBM, int GF>
@@ -1133,7 +1136,7 @@ __global__ __launch_bounds__(Shape<TBM>::W * 64) void k_gemm_down_p(GemmArgs a) 
     static_assert(TBM >= 2, "persistent kernels take 32- and 80-row tiles");
     __shared__ __attribute__((aligned(16))) _Float16 xs[3 * Shape<TBM>::XR * BLD];
     __shared__ int rowoff[3 * TBM * 16];
-    tile_stream<EFMT, 1, DN_RPW, Shape<TBM>::DEPTH, 4, TBM>(DnPol{a}, xs, rowoff);
+    tile_stream<EFMT, 1, DN_RPW, Shape<TBM>::DEPTH, 4, TBM>(DnPol<>{a}, xs, rowoff);
 }
 
 /* Routed and shared matrices of two tile-major formats in one launch: a
@@ -1151,7 +1154,6 @@ DEV void two_walks(const GemmArgs &a, GemmArgs &ar, GemmArgs &as) {
     as = a;
     ar.uwin = -a.nsh;
     as.uwin = a.nsh;
-    as.urev = 1;
 }
 template <int TBM>
 __global__ __launch_bounds__(Shape<TBM>::W * 64) void k_gemm_down_p2(GemmArgs a) {
@@ -1161,15 +1163,15 @@ __global__ __launch_bounds__(Shape<TBM>::W * 64) void k_gemm_down_p2(GemmArgs a)
     __shared__ int rowoff[3 * TBM * 16];
     GemmArgs ar, as;
     two_walks(a, ar, as);
-#define WALK(F, ARGS) tile_stream<F, 1, DN_RPW, Shape<TBM>::DEPTH, 4, TBM>(DnPol{ARGS}, xs, rowoff)
-    if (a.fmt == FQ4KT) WALK(FQ4KT, ar);
-    else if (a.fmt == FQ5KT) WALK(FQ5KT, ar);
-    else WALK(FQ6KT, ar); /* (the launcher sends no other routed format) */
+#define WALK(F, REV, ARGS) tile_stream<F, 1, DN_RPW, Shape<TBM>::DEPTH, 4, TBM>(DnPol<REV>{ARGS}, xs, rowoff)
+    if (a.fmt == FQ4KT) WALK(FQ4KT, false, ar);
+    else if (a.fmt == FQ5KT) WALK(FQ5KT, false, ar);
+    else WALK(FQ6KT, false, ar); /* (the launcher sends no other routed format) */
     __syncthreads();
-    if (a.fmt_sh == FQ4KT) WALK(FQ4KT, as);
-    else if (a.fmt_sh == FQ5KT) WALK(FQ5KT, as);
-    else if (a.fmt_sh == FQ6KT) WALK(FQ6KT, as);
-    else WALK(FQ8T, as);
+    if (a.fmt_sh == FQ4KT) WALK(FQ4KT, true, as);
+    else if (a.fmt_sh == FQ5KT) WALK(FQ5KT, true, as);
+    else if (a.fmt_sh == FQ6KT) WALK(FQ6KT, true, as);
+    else WALK(FQ8T, true, as);
 #undef WALK
 }
 template <int TBM>
@@ -1180,9 +1182,9 @@ __global__ __launch_bounds__(Shape<TBM>::W * 64) void k_gemm_gate_up_p2(GemmArgs
     KT_BEGIN(a.kt);
     GemmArgs ar, as;
     two_walks(a, ar, as);
-    tile_stream<FQ4KT, 2, GU_RPW, Shape<TBM>::DEPTH, 16, TBM>(GuPol{ar}, xs, rowoff);
+    tile_stream<FQ4KT, 2, GU_RPW, Shape<TBM>::DEPTH, 16, TBM>(GuPol<>{ar}, xs, rowoff);
     __syncthreads();
-    tile_stream<FQ8T, 2, GU_RPW, 2, 16, TBM>(GuPol{as}, xs, rowoff);
+    tile_stream<FQ8T, 2, GU_RPW, 2, 16, TBM>(GuPol<true>{as}, xs, rowoff);
     KT_END(a.kt);
 }
 
