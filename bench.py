@@ -269,9 +269,11 @@ def run_config(key, steps, warmup, path, cpu_seconds, no_cpu, graph=True):
     gu_us = stage_us["gate_up"]
     gu_gbs = gu_bytes / (gu_us * 1e-6) / 1e9
     gu_tflops = gu_flops / (gu_us * 1e-6) / 1e12
-    # up to T K = 32 E every expert is in 32-row tiles (one list), above 44 E
-    # in 80-row tiles, between them in both lists
+    # the stage events' eager launches: up to T K = 32 E every expert is in
+    # 32-row tiles (one list), above 44 E in 80-row tiles, between them in both
+    # lists; a captured call takes both lists above 44 E too
     both_lists = 32 * E < T * K <= 44 * E
+    big_eagerly = kpath == "mfma" and graph and T * K > 44 * E
     kname = {"gemv": "gemv_gate_up", "small_batch_gemm": "gemm_gate_up (16-row tiles)",
              "mfma": ("gemm_gate_up (32-row tile list)" if T * K <= 32 * E
                       else "gemm_gate_up (32-row + 80-row tile lists)" if both_lists
@@ -298,7 +300,10 @@ def run_config(key, steps, warmup, path, cpu_seconds, no_cpu, graph=True):
                            "(%d launches)%s" % (n_prof * nl,
                                                 "; under stage timing the two tile lists run one after the "
                                                 "other on one stream, where the timed steps overlap them on two"
-                                                if serial else ""),
+                                                if serial else
+                                                "; these eager launches take one 80-row tile list, where the "
+                                                "timed graph runs a 32-row and an 80-row list on two streams"
+                                                if big_eagerly else ""),
                  "in_kernel_us": round(float(np.mean(spans)), 3),
                  "gbs": round(gu_gbs, 1), "tflops": round(gu_tflops, 2)})
     if rp.get("rocprof_gate_up_avg_us"):

@@ -692,11 +692,12 @@ static int forward_impl(orome_hip_ctx *c, const OromeHipModelConfig *cfg, const 
             a.x16 = NULL;
             TLAUNCH(c, ST_TOPK, launch_topk(a, s), "top-k");
         }
+        const int lists = gemm_lists(T, K, E, s);
+        a.lists = lists;
         if (!self_dispatch)
             TLAUNCH(c, ST_DISPATCH, launch_dispatch(a, c->tiles, c->tiles_b, S ? 1 : 0, c->dcount, s, a.dcnt ? 1 : 0), "dispatch");
         const GemmSelfDispatch sdargs = {c->dcount, dispatch_blocks(T), c->tmask, c->idx, c->offsets, c->pairs, c->pos};
         /* one launch per tile list (grid sized for the most tiles it can hold) */
-        const int lists = gemm_lists(T, K, E);
         const bool sh_small = lists == LISTS_SMALL;
         const int ns_max = E + (sh_small ? (T * K) / GEMM_TILE_SMALL : 0) +
                            (S && sh_small ? (T + GEMM_TILE_SMALL - 1) / GEMM_TILE_SMALL : 0),

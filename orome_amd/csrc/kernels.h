@@ -73,6 +73,7 @@ struct RouteArgs {
      * tile list (one tile per active expert, then the shared expert's) */
     uint32_t *tiles_s;
     int has_shared;
+    int lists;           /* the tile lists the dispatch writes (gemm_lists) */
     /* exact top-k above the one-block dispatch's size: also adds each
      * selected (token, expert) to dcnt[token / 256][expert], the counts the
      * three-launch dispatch would otherwise count (launch_dispatch(counted));
@@ -207,14 +208,21 @@ int launch_fill_u32(void *p, uint32_t v, size_t words, hipStream_t s);
  *   LISTS_BOTH    experts with <= GEMM_TILE_SMALL rows one small tile each,
  *                 the rest and the shared expert tiles of GEMM_TILE_BIG, the
  *                 big list on a second stream beside the small one;
- *   LISTS_BIG (T*K > GEMM_BIG_ONLY E)  every expert in tiles of
- *                 GEMM_TILE_BIG: the few small experts cost less there than a
- *                 nearly empty pair of launches and the two streams' fork and
- *                 join (~20 us a layer launched eagerly).  Layers of 256
- *                 experts, K = 8, both lists -> big only: T = 2048 317 -> 293
- *                 us, 1500 293 -> 271, 4096 613 -> 591; 1300 (40 rows an
- *                 expert) 765 -> 766 for three layers; 1100 (34 rows) 239 ->
- *                 250.
+ *   LISTS_BIG (T*K > GEMM_BIG_ONLY E, launched eagerly)  every expert in
+ *                 tiles of GEMM_TILE_BIG, one list on the caller's stream.
+ * What LISTS_BIG saves is the second pair of launches and the two streams'
+ * fork and join; what it costs is five token blocks for an expert of a few
+ * rows.  Both lists -> big only, E = 256, K = 8, us a layer:
+ *   eager, balanced   1500 285 -> 264, 2048 309 -> 287, 4096 556 -> 534
+ *   eager, Zipf 1.1   1500 256 -> 235, 2048 292 -> 286, 4096 537 -> 525
+ *   captured, balanced  1500 265 -> 265, 2048 292 -> 288, 4096 543 -> 536
+ *   captured, Zipf 1.1  1500 229 -> 237, 2048 276 -> 287, 4096 508 -> 523
+ * (of 109 experts in use at 2048 under Zipf, 73 hold at most 32 rows).  In a
+ * graph the fork and join cost a few us, so a captured call keeps both lists:
+ * big only loses 3-4 % there under skew (6 % at 128 experts, 13 % at 64) for
+ * 0-2 % of balanced routing.  Eagerly, wider layers of 64 or 128 experts gain
+ * 5-12 % balanced and -4 to +17 % under skew.  Below 44 rows an expert both
+ * lists win eagerly too (1100 tokens, 34 rows: 239 against 250).
  * Capacities: small 2E + T/SMALL + 1, big T*K/BIG + E + T/BIG + 1. */
 enum { LISTS_SMALL, LISTS_BOTH, LISTS_BIG };
 #define GEMM_BIG_ONLY 44
@@ -225,7 +233,10 @@ enum { LISTS_SMALL, LISTS_BOTH, LISTS_BIG };
 #ifndef GEMM_TILE_BIG
 #define GEMM_TILE_BIG 80
 #endif
-static inline __host__ __device__ int gemm_lists(int T, int K, int E) {
-    const long tk = (long)T * K;
-    return tk <= (long)GEMM_TILE_SMALL * E ? LISTS_SMALL : tk > (long)GEMM_BIG_ONLY * E ? LISTS_BIG : LISTS_BOTH;
+static inline bool gemm_lists_small(int T, int K, int E) { return (long)T * K <= (long)GEMM_TILE_SMALL * E; }
+static inline int gemm_lists(int T, int K, int E, hipStream_t s) {
+    if (gemm_lists_small(T, K, E)) return LISTS_SMALL;
+    if ((long)T * K <= (long)GEMM_BIG_ONLY * E) return LISTS_BOTH;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(s, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone ? LISTS_BIG : LISTS_BOTH;
 }

@@ -1254,8 +1254,7 @@ int gemm_small_tiles_ok(const ExpertSide &ex, const SharedSide &sh, int H, int M
 static int shared_tiles_in(const SharedSide &sh, int T, int K, int E, int tile_m) {
     if (!sh.gate) return 0;
     if (tile_m == GEMM_TILE_MIN) return 1; /* small-batch list: T <= 16, one shared tile */
-    const bool sh_small = gemm_lists(T, K, E) == LISTS_SMALL;
-    return (tile_m == GEMM_TILE_SMALL) == sh_small ? (T + tile_m - 1) / tile_m : 0;
+    return (tile_m == GEMM_TILE_SMALL) == gemm_lists_small(T, K, E) ? (T + tile_m - 1) / tile_m : 0;
 }
 
 #ifndef GEMM_SELF_DISPATCH

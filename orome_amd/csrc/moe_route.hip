@@ -608,7 +608,7 @@ DEV void dispatch_lists(const RouteArgs &a, uint32_t c, uint32_t *xo, uint32_t *
     /* glob false: the exclusive offsets into xo only (the blocks of a
      * dispatch that one other block writes the lists for) */
     const int E = a.E, T = a.T, tid = threadIdx.x;
-    const int lists = gemm_lists(T, a.K, E);
+    const int lists = a.lists;
     const bool so = lists == LISTS_SMALL, mine = tid < E;
     if (!mine) c = 0;
     const uint32_t ns_own = n_small_tiles(c, lists), nb_own = n_big_tiles(c, lists);

@@ -2,6 +2,8 @@
 top-k, LDS counting-sort dispatch, MFMA grouped GEMMs, combine) against the
 C oracle.  Expert indices and dispatch order bit-exact; outputs within 1e-3
 relative L2 (fp16 weight tiles: expected ~1e-4)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -9,7 +11,7 @@ import orome_amd
 import oracle as O
 from conftest import banner
 from orome_amd import _lib
-from orome_amd._lib import lib
+from orome_amd._lib import check, lib
 from orome_amd.moe import DeviceBuffer
 from test_gpu_decode import Pair, assert_logits, rel_l2
 
@@ -574,4 +576,53 @@ def test_routed_and_shared_formats_in_one_launch(T, down, shared, shared_down):
     p.gm.unpack()
     plain, _ = p.run(0, x, h, K=4, path=_lib.OROME_PATH_MFMA)
     assert np.array_equal(out, plain)
+    p.gm.close()
+
+
+@pytest.mark.parametrize("kw", [dict(), dict(zipf=True, down=14, shared=8), dict(H=3072, zipf=True)])
+def test_tile_lists_of_a_captured_call(kw):
+    """Above 44 rows an expert an eager call puts every expert in 80-row tiles
+    and a captured one keeps the 32-row list beside them (its gate/up stamps
+    fill the second half of the stamp buffer): the same bits, replay after
+    replay with eager calls between them."""
+    banner("captured tile lists %s" % kw)
+    T, K, nb = 300, 4, 16384
+    p = Pair(max_tokens=T, **{**dict(H=2048, E=16, M=512, S=512, seed=92), **kw})
+    x, h = p.inputs(T, seed=6200)
+    dx, dh, do = DeviceBuffer.from_array(p.ctx, x), DeviceBuffer.from_array(p.ctx, h), DeviceBuffer(p.ctx, h.nbytes)
+    buf = DeviceBuffer(p.ctx, nb * 2 * 8)
+    zeros = np.zeros(nb * 2, np.uint64)
+
+    def stamps():
+        v = buf.download(np.uint64, (2, nb // 2, 2))[..., 0] > 0
+        buf.upload(zeros)
+        return int(v[0].sum()), int(v[1].sum())
+
+    buf.upload(zeros)
+    check(lib.orome_hip_kernel_timing(p.ctx.handle, buf.ptr, nb), "kernel_timing")
+    try:
+        p.gm.forward(0, dx, dh, do, T, K)
+        p.ctx.sync()
+        eager = do.download(np.float32, h.shape)
+        big, small = stamps()
+        assert big and not small
+        check(lib.orome_hip_capture_begin(p.ctx.handle))
+        p.gm.forward(0, dx, dh, do, T, K)
+        ex = C.c_void_p()
+        check(lib.orome_hip_capture_end(p.ctx.handle, C.byref(ex)))
+        for rep in range(3):
+            do.upload(np.zeros_like(h))
+            check(lib.orome_hip_graph_launch(p.ctx.handle, ex))
+            p.ctx.sync()
+            assert np.array_equal(do.download(np.float32, h.shape), eager), "replay %d" % rep
+            big, small = stamps()
+            assert big and small
+            p.gm.forward(0, dx, dh, do, T, K)
+            p.ctx.sync()
+            assert np.array_equal(do.download(np.float32, h.shape), eager)
+            stamps()
+        check(lib.orome_hip_graph_destroy(ex))
+    finally:
+        check(lib.orome_hip_kernel_timing(p.ctx.handle, None, 0), "kernel_timing")
+    buf.free()
     p.gm.close()
