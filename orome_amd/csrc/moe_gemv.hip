@@ -233,7 +233,11 @@ struct GUArgs {
  * i + step, i + 2 step, ... (< H / 8) of a row-major matrix, the pair
  * starting at group slot s0: the rows that the T = 1 down kernel's blocks g
  * read, from a block on the same XCD as they are (g = i mod 8).  The value
- * lands in `sink`, which the caller keeps until a wait for it. */
+ * lands in `sink`, which the caller keeps until a wait for it.  64 lanes hold
+ * two groups of up to 32 lines (Q4_K, Q5_K and Q6_K rows of 512: 18, 22, 27);
+ * a Q8_0 group of such rows has 34, and the last 4 lines of the second one
+ * are left to the next kernel: with a third wave touching them a call takes
+ * the same 16.3 us (and 0-1.5 % longer beside a Q5_K down). */
 DEV void touch_rows8(const uint8_t *m, int rb, int H, int i, int step, int s0, int lane, uint32_t &sink) {
     const int nl = (8 * rb + 127) / 128, g = i + step * (s0 + lane / nl);
     if (lane / nl >= 2 || g >= H / 8) return;
@@ -435,8 +439,8 @@ DEV void k_gemv_gate_up1_body(GUArgs a, RouteArgs ra) {
         const float Xl = cvt_x16_f32(xr, xs), Xh = cvt_x16_f32(xr + 4, xs + 8);
         const int r0 = (b - a.routed_blocks) * rows_blk + wv * GU_RPW;
         uint32_t sink = 0;
-        /* waves 1 and 2 touch the group slots 0..3 of this block's rows (the
-         * H / 8 groups of 8 rows over S / (4 GU_RPW) blocks: 4 each at
+        /* waves 1 and 2 touch the group slots 0..3 of this block's rows (but
+         * for a few lines of Q8_0 rows; the H / 8 groups of 8 rows over S / (4 GU_RPW) blocks: 4 each at
          * H = 2048, S = 512) */
         if ((wv == 1 || wv == 2) && a.pf_sh_down)
             touch_rows8(a.pf_sh_down, a.pf_sh_rb, a.H, b - a.routed_blocks, a.S / rows_blk, 2 * (wv - 1), lane, sink);
