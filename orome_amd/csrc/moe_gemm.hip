@@ -1050,21 +1050,21 @@ DEV void k_gemm_gate_up_body(GemmArgs a) {
             lds_barrier();
         }
     };
-    constexpr bool NT = (TBM >= 5 || TBM == 1) && TILED(RF);
+    constexpr bool ONCE = TBM >= 5 || TBM == 1; /* no other tile reads these weights */
     /* a 32-row tile holding at most 16 rows runs the 16-row code: half the
      * matrix instructions and B-fragment reads, the same weight stream */
     if (sh) {
         const GuEpi epi{a.act_sh, a.S, (int)first, (int)rows};
         constexpr int D = SF == FQ8 || SF == FQ8T ? 2 : Shape<TBM>::DEPTH;
         if (TBM == 2 && rows <= 16)
-            tile_run<SF, 2, GU_RPW, D, NST, 1, NT>(a.sh_a, a.sh_b, a.H, a.src, a.H, rowoff, (int)rows, yb, xs, epi, fill);
-        else tile_run<SF, 2, GU_RPW, D, NST, TBM, NT>(a.sh_a, a.sh_b, a.H, a.src, a.H, rowoff, (int)rows, yb, xs, epi, fill);
+            tile_run<SF, 2, GU_RPW, D, NST, 1, ONCE && TILED(SF)>(a.sh_a, a.sh_b, a.H, a.src, a.H, rowoff, (int)rows, yb, xs, epi, fill);
+        else tile_run<SF, 2, GU_RPW, D, NST, TBM, ONCE && TILED(SF)>(a.sh_a, a.sh_b, a.H, a.src, a.H, rowoff, (int)rows, yb, xs, epi, fill);
     } else {
         const GuEpi epi{a.act, a.M, (int)first, (int)rows};
         const uint8_t *w0 = a.wa + (size_t)e * a.stride_a, *w1 = a.wb + (size_t)e * a.stride_b;
         if (TBM == 2 && rows <= 16)
-            tile_run<RF, 2, GU_RPW, Shape<TBM>::DEPTH, NST, 1, NT>(w0, w1, a.H, a.src, a.H, rowoff, (int)rows, yb, xs, epi, fill);
-        else tile_run<RF, 2, GU_RPW, Shape<TBM>::DEPTH, NST, TBM, NT>(w0, w1, a.H, a.src, a.H, rowoff, (int)rows, yb, xs, epi, fill);
+            tile_run<RF, 2, GU_RPW, Shape<TBM>::DEPTH, NST, 1, ONCE && TILED(RF)>(w0, w1, a.H, a.src, a.H, rowoff, (int)rows, yb, xs, epi, fill);
+        else tile_run<RF, 2, GU_RPW, Shape<TBM>::DEPTH, NST, TBM, ONCE && TILED(RF)>(w0, w1, a.H, a.src, a.H, rowoff, (int)rows, yb, xs, epi, fill);
     }
 }
 
