@@ -1105,11 +1105,9 @@ __global__ __launch_bounds__(Shape<TBM>::W * 64) void k_gemm_down(GemmArgs a) {
 #ifndef GEMM_PERSIST
 #define GEMM_PERSIST 1
 #endif
-/* small tiles: 0 = per-tile kernels, n = persistent with n blocks per CU
- * (measured: the down projection gains ~10 % at T = 512, gate/up nothing) */
-#ifndef GEMM_PERSIST_SMALL
-#define GEMM_PERSIST_SMALL 0
-#endif
+/* the down projection's small tiles: 0 = per-tile kernels, n = persistent
+ * with n blocks per CU (measured: ~10 % at T = 512; the gate/up gained
+ * nothing and keeps per-tile kernels) */
 #ifndef GEMM_PERSIST_SMALL_DN
 #define GEMM_PERSIST_SMALL_DN 2
 #endif
@@ -1118,7 +1116,7 @@ DEV void k_gemm_gate_up_p_body(GemmArgs a) {
     static_assert(TBM >= 2, "persistent kernels take 32- and 80-row tiles");
     __shared__ __attribute__((aligned(16))) _Float16 xs[3 * Shape<TBM>::XR * BLD];
     __shared__ int rowoff[3 * TBM * 16];
-    tile_stream<GF, 2, GU_RPW, (GF == FQ8 || GF == FQ8T ? 2 : Shape<TBM>::DEPTH), 16, TBM>(GuPol<>{a}, xs, rowoff);
+    tile_stream<GF, 2, GU_RPW, (GF == FQ8 ? 2 : Shape<TBM>::DEPTH), 16, TBM>(GuPol<>{a}, xs, rowoff);
 }
 
 template <int TBM, int GF>
@@ -1262,7 +1260,7 @@ static int shared_tiles_in(const SharedSide &sh, int T, int K, int E, int tile_m
 #endif
 bool gemm_self_dispatch_ok(int T, int K, int E) {
     const long tk = (long)T * K;
-    return GEMM_SELF_DISPATCH && !GEMM_PERSIST_SMALL && E <= 256 && T <= 1024 && tk <= (long)GEMM_TILE_SMALL * E;
+    return GEMM_SELF_DISPATCH && E <= 256 && T <= 1024 && tk <= (long)GEMM_TILE_SMALL * E;
 }
 
 int launch_gemm_gate_up(const ExpertSide &ex, const SharedSide &sh, const _Float16 *x16, int zrow, int T,
@@ -1297,29 +1295,23 @@ int launch_gemm_gate_up(const ExpertSide &ex, const SharedSide &sh, const _Float
     }
     const dim3 grid((unsigned)((n_tiles_max + 7) / 8 * 8 * a.nyb)), block(W * 64);
     const bool q8 = sh.gate && (sh.gate_fmt == FQ8 || sh.gate_fmt == FQ8T);
-    const unsigned pb = !GEMM_PERSIST || tile_m == GEMM_TILE_MIN ? 0u
-                        : tile_m == GEMM_TILE_BIG ? persist_blocks() : GEMM_PERSIST_SMALL * persist_blocks();
+    const unsigned pb = GEMM_PERSIST && tile_m == GEMM_TILE_BIG ? persist_blocks() : 0u;
     a.kt = kt && (long)grid.x <= kt_cap ? kt : nullptr;
     if (pb && H == 2048 && (!sh.gate || sh.S == M)) {
         a.kt = kt && (long)pb <= kt_cap ? kt : nullptr;
-#define GP_LAUNCH(GF, ARGS)                                                                                      \
-    do {                                                                                                         \
-        if (tile_m == GEMM_TILE_BIG) KLAUNCH((k_gemm_gate_up_p<GEMM_TILE_BIG / 16, GF>), dim3(pb), block, 0, s, ARGS); \
-        else KLAUNCH((k_gemm_gate_up_p<GEMM_TILE_SMALL / 16, GF>), dim3(pb), block, 0, s, ARGS);          \
-    } while (0)
+#define GP_LAUNCH(GF, ARGS) KLAUNCH((k_gemm_gate_up_p<GEMM_TILE_BIG / 16, GF>), dim3(pb), block, 0, s, ARGS)
         const int nsh = shared_tiles_in(sh, T, K, E, tile_m);
-        if (nsh && tiled && sh.gate_fmt == FQ8T && tile_m == GEMM_TILE_BIG) { /* Q8_0 shared expert: two walks */
+        if (nsh && sh.gate_fmt == FQ8T) { /* Q8_0 shared expert: two walks */
             a.nsh = nsh;
             KLAUNCH((k_gemm_gate_up_p2<GEMM_TILE_BIG / 16>), dim3(pb), block, 0, s, a);
-        } else if (nsh && q8) { /* (a launch for the routed tiles, one for the shared) */
+        } else if (nsh && q8) { /* (row-major: a launch for the routed tiles, one for the shared) */
             GemmArgs ar = a, as = a;
             ar.uwin = -nsh;
             as.uwin = nsh;
             as.kt = nullptr;
             if (tiled) GP_LAUNCH(FQ4KT, ar);
             else GP_LAUNCH(FQ4K, ar);
-            if (sh.gate_fmt == FQ8T) GP_LAUNCH(FQ8T, as);
-            else GP_LAUNCH(FQ8, as);
+            GP_LAUNCH(FQ8, as);
         } else if (tiled) {
             GP_LAUNCH(FQ4KT, a);
         } else {
