@@ -146,7 +146,7 @@ def test_persistent_gemm_zipf_q6k(monkeypatch, shared_down):
     """Skewed routing (a few experts with many tiles, many with none) and a
     Q6_K down projection through a 16-block persistent grid, against the
     oracle and bit-identical to the per-tile kernels.  With a Q4_K shared
-    down the routed and shared tiles are walked by two launches."""
+    down each block walks its routed tiles, then its shared ones."""
     banner("persistent GEMM, Zipf T=512, Q6_K down, shared down type %d" % shared_down)
     p = Pair(max_tokens=512, down=14, shared_down=shared_down, zipf=True, seed=35)
     monkeypatch.setenv("OROME_GEMM_PERSIST_BLOCKS", "16")
@@ -529,12 +529,13 @@ def test_gate_up_stage_counts(H, shared):
     """The gate/up loop over a run-time stage count (every H but 2048): one
     pass (H = 512: two activation chunks, both resident), odd numbers of
     passes and the largest size, on 16- and 32-row tiles (T = 9, 70) and
-    80-row ones (T = 260, K T > 32 E), with a Q4_K and a Q8_0 shared expert.
+    80-row ones (beside 32-row ones at T = 150, alone at T = 260), with a Q4_K
+    and a Q8_0 shared expert.
     Each equals its unpacked run bit for bit (row-major spans, the same loop)
     and the oracle within tolerance."""
     banner("gate/up stage counts, H=%d shared=%d" % (H, shared))
     p = Pair(max_tokens=260, H=H, E=16, M=256, S=256, shared=shared, seed=H)
-    for T in (9, 70, 260):
+    for T in (9, 70, 150, 260):
         out, _ = run_and_check(p, T, seed=5000 + T, K=4)
         x, h = p.inputs(T, seed=5000 + T)
         p.gm.unpack()
@@ -563,19 +564,26 @@ def test_tile_lists_at_their_limits(T, kw):
     p.gm.close()
 
 
-@pytest.mark.parametrize("T", [129, 177, 300])
+@pytest.mark.parametrize("T", [128, 129, 177, 300])
 @pytest.mark.parametrize("down,shared,shared_down", [(12, 8, 8), (12, 12, 13), (13, 8, 12), (13, 12, 14), (14, 12, 13), (14, 8, 8)])
-def test_routed_and_shared_formats_in_one_launch(T, down, shared, shared_down):
+def test_routed_and_shared_formats_in_one_launch(monkeypatch, T, down, shared, shared_down):
     """Q4_K / Q5_K / Q6_K routed down matrices beside a shared expert in
     another format: the packed layer walks both in one launch and has to equal,
-    bit for bit, the unpacked one (a launch each)."""
+    bit for bit, the unpacked one (a launch each).  32-row tiles at T = 128,
+    80-row ones above; on the full grid, where a block makes one walk or the
+    other, and on one block per XCD, where those of the first XCDs walk several
+    routed units and then several shared ones."""
     banner("two walks T=%d %d %d %d" % (T, down, shared, shared_down))
     p = Pair(max_tokens=300, H=2048, E=16, M=512, S=512, seed=91, down=down, shared=shared, shared_down=shared_down)
     out, _ = run_and_check(p, T, seed=6100 + T, K=4)
     x, h = p.inputs(T, seed=6100 + T)
+    monkeypatch.setenv("OROME_GEMM_PERSIST_BLOCKS", "8")
+    few, _ = p.run(0, x, h, K=4, path=_lib.OROME_PATH_MFMA)
+    monkeypatch.delenv("OROME_GEMM_PERSIST_BLOCKS")
     p.gm.unpack()
     plain, _ = p.run(0, x, h, K=4, path=_lib.OROME_PATH_MFMA)
     assert np.array_equal(out, plain)
+    assert np.array_equal(few, plain)
     p.gm.close()
 
 
