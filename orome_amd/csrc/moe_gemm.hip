@@ -1142,10 +1142,10 @@ __global__ __launch_bounds__(Shape<TBM>::W * 64) void k_gemm_down_p(GemmArgs a) 
  * (they end the list), which are dealt from the other end of each XCD's
  * blocks, first to those that had a routed unit less.  As two launches the
  * second one's few units ran alone, about one a CU, behind the first one's
- * last round.  Layer speed against one earlier build, two launches -> one:
- * 4096 tokens with a Q6_K down and a Q4_K shared one 1.044 -> 1.066 (about
- * 12 us of 572), 777 tokens with Q5_K and a Q8_0 shared expert 1.002 ->
- * 1.023, 512 with skewed routing and a Q6_K down 1.003 -> 1.027.  (Row-major
+ * last round.  Whole layers, two launches -> one: 2048 tokens with a Q6_K
+ * down and a Q4_K shared one 330 -> 315 us, with Q5_K and a Q8_0 shared expert
+ * (its gate/up too) 346 -> 312, 4096 with Q6_K 596 -> 581, 777 with Q5_K and
+ * Q8_0 195 -> 192, 512 with skewed routing and Q6_K 132 -> 129.  (Row-major
  * layers keep a launch each: their Q8_0 walk spills registers by itself.) */
 DEV void two_walks(const GemmArgs &a, GemmArgs &ar, GemmArgs &as) {
     ar = a;
